@@ -271,7 +271,7 @@ dbi_status check_chunk(const dbi_kv* kv, uint32_t pos0, uint32_t n) {
 
 // workspace of a chunk call (no launch)
 dbi_status chunk_prepare(dbi_kv* kv, const dbi::AttnCall& c, bool* prefill) {
-  *prefill = dbi::prefill_supported(kv->geom, c.n_heads, c.rows);
+  *prefill = dbi::prefill_supported(kv->geom, c);
   if (*prefill) return ensure_part(kv, dbi::prefill_workspace_need(kv->geom, c));
   return ensure_workspace(kv, c);
 }
@@ -926,7 +926,7 @@ dbi_status dbi_attn_splits(const dbi_kv* kv, uint32_t pos0, uint32_t rows, uint3
   if (dbi_status st = check_rows(kv, pos0, rows)) return st;
   dbi::AttnCall c = chunk_call(0, pos0, rows, n_heads, 1.0f, nullptr, nullptr);
   if (kv->geom.ring) c.ring = ring_view(kv, pos0 + 1);
-  const bool pre = dbi::prefill_supported(kv->geom, c.n_heads, c.rows);
+  const bool pre = dbi::prefill_supported(kv->geom, c);
   *n_split = static_cast<uint32_t>(pre ? dbi::prefill_split_count(kv->geom, c)
                                        : dbi::attention_split_count(kv->geom, c));
   return DBI_OK;

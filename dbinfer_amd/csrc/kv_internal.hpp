@@ -196,13 +196,15 @@ hipError_t launch_attention(const KvGeom& g, const KvStore& s, Workspace& ws,
 // Number of partial floats one call needs (for workspace sizing).
 size_t attention_workspace_need(const KvGeom& g, const AttnCall& c);
 
-// Causal chunks of at least this many rows over the dense fp32 cache run on
-// the matrix cores (prefill.hip); shorter ones (verify rounds) through
-// launch_attention, whose many small per-wave streams keep more bytes in
-// flight than the prefill kernel's one staged stream per workgroup.
+// Causal chunks of at least this many rows over the dense fp32 cache may run
+// on the matrix-core prefill kernel (prefill.hip); shorter ones (verify
+// rounds) go through launch_attention, whose many small per-wave streams keep
+// more bytes in flight than the prefill kernel's one staged stream per
+// workgroup. prefill_supported decides by the chunk's size.
 constexpr int kPrefillMinRows = 64;
-constexpr int kPrefillMaxSplits = 8;  // key splits of one chunk (workspace records)
-bool prefill_supported(const KvGeom& g, int n_heads, int rows);
+constexpr int kPrefillMaxSplits = 32;  // key splits of one row block
+constexpr int kPrefillBlocks = 256;    // workgroups of a launch that splits keys (one per CU)
+bool prefill_supported(const KvGeom& g, const AttnCall& c);
 size_t prefill_workspace_need(const KvGeom& g, const AttnCall& c);
 hipError_t launch_prefill(const KvGeom& g, const KvStore& s, Workspace& ws, const AttnCall& c,
                           hipStream_t st);
