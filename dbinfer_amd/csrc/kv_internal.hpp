@@ -196,7 +196,7 @@ hipError_t launch_attention(const KvGeom& g, const KvStore& s, Workspace& ws,
 // Number of partial floats one call needs (for workspace sizing).
 size_t attention_workspace_need(const KvGeom& g, const AttnCall& c);
 
-// Causal chunks of at least this many rows over the dense fp32 cache may run
+// Causal chunks of at least this many rows over a dense cache may run
 // on the matrix-core prefill kernel (prefill.hip); shorter ones (verify
 // rounds) go through launch_attention, whose many small per-wave streams keep
 // more bytes in flight than the prefill kernel's one staged stream per

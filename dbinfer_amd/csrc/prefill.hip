@@ -1,4 +1,4 @@
-// Causal chunk attention of the dense fp32 cache on the matrix cores: the
+// Causal chunk attention of the dense caches on the matrix cores: the
 // attention loop of decode_layer_chunk (model.cpp:956-981), rows c of a
 // chunk at pos0 attending keys [0, pos0 + c], for chunks long enough to
 // make QK^T and PV real matrix products (the prefill chunks of config 2).
@@ -30,6 +30,16 @@
 //    sinks to about 1.5 GHz under the products of hd 128 (the matrix units
 //    busy 90 % of the time then), which is what a large bf16 matrix product
 //    reaches too (1.3 PFLOP/s).
+//  - Dense int8: the staging dequantizes, k = fp32(code * scale) per channel
+//    and v = fp32(code * scale) per 32-channel block, and takes the fp32 sinks
+//    for positions < n_sink; everything after it is the fp32 kernel. One fp32
+//    rounding of code * scale stands where attend_dense_int8 (model.cpp:
+//    605-660) rounds q * scale and weight * scale, so the error against 64
+//    bits is of the same size (256 rows of 24/8 heads at 3840, hd 128: 5.8e-7,
+//    7.0e-7 with the products of codes). Exact products of codes would halve
+//    the matrix work, but need the query scaled and split per 32-key group,
+//    about 300 vector instructions per stage and 16 vectors, which is what
+//    bounds the rows kernel (that chunk 98 us there, 81 here).
 //  - Key splits: the row blocks' stages are dealt to workgroups of at most T
 //    stages each, T the smallest that needs at most one workgroup per CU
 //    (prefill_plan), so a causal chunk's longer row blocks get more of them.
@@ -71,6 +81,16 @@ constexpr int kMaxItems = kPrefillBlocks;
 struct PrefillParams {
   const float* kf;  // this layer's K, V: [nkv][capg * hd], granule layout
   const float* vf;
+  // dense int8: codes [nkv][capg * hd] in the matrix-core layout, K channel
+  // scales [nkv][ng][hd], V block scales [nkv][capg][hd / 32], sinks
+  // [nkv][n_sink][hd]
+  const int8_t* k8;
+  const int8_t* v8;
+  const float* ks;
+  const float* vs;
+  const float* ksink;
+  const float* vsink;
+  int ng, n_sink;
   const float* q;   // [rows][n_heads][hd]
   float* out;       // [rows][n_heads][hd]
   float* part;      // split records, one region of record_floats per workgroup
@@ -140,7 +160,7 @@ __device__ __forceinline__ f32x16 mfma32(const uint4& a, const uint4& b, const f
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-template <int HD>
+template <int HD, bool I8>
 __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_kernel(const PrefillParams P) {
   using S = Stage<HD>;
   constexpr int SK = S::SK, UPR = S::UPR, PLANE = S::PLANE, BUF = S::BUF, NU = S::NU;
@@ -192,8 +212,6 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
   const int wave_last = P.pos0 + min(row0 + RPV - 1, P.rows - 1);  // wave-uniform
 
   const size_t head_el = static_cast<size_t>(kh) * P.capg * HD;
-  const float* kbase = P.kf + head_el;
-  const float* vbase = P.vf + head_el;
 
   // ---- staging. K lanes (the first half of the waves, t < STG): units
   // u = t + STG m, key u / UPR, dims 8 (u % UPR) .. + 7 (two float4 of the
@@ -209,32 +227,81 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
   // LDS, its swizzle the same). V: key e's dims (e & 3) row pieces of 16
   // bytes x HD/8 and (e >> 2) times 8 keys of a granule (1024 / (HD/64) floats
   // x NU = HD/64: 32 HD bytes) on; output row m 32 units.
-  uint32_t src, dst;
+  // int8: K: a unit is 8 consecutive bytes, unit m one granule (16 HD bytes)
+  // on, its 8 channel scales shared; V: a dim's keys 0..3 are 4 bytes, keys
+  // 8..11 512 bytes on, the next dim 16 bytes on; scl the scale of the first
+  // key, HD/32 floats apart.
+  uint32_t src, dst, scl = 0;
+  int vd = 0;  // V: the lane's first dim
   const int kq = (wave - kPWaves / 2) & 3;              // V: k-step and lane half
   const int vkey0 = 16 * (kq >> 1) + 4 * (kq & 1);      // V: keys vkey0 + {0..3, 8..11}
   if (k_stager) {
     const int key = static_cast<int>(threadIdx.x) / UPR, u = static_cast<int>(threadIdx.x) % UPR;
-    src = static_cast<uint32_t>(k_off_tiled(HD, false, key, 8 * u)) * 4u;
+    src = I8 ? static_cast<uint32_t>(k_off_i8d(HD, key, 8 * u))
+             : static_cast<uint32_t>(k_off_tiled(HD, false, key, 8 * u)) * 4u;
+    scl = 8u * u * 4u;
     dst = static_cast<uint32_t>((key * UPR + (u ^ kswz<HD>(key))) * 16);
   } else {
     const int c = lane, r5 = c & 31;
     const int d = ((r5 >> 2) & 1) * (HD / 2) + (c >> 5) * 16 * NU + (4 * (r5 >> 3) + (r5 & 3)) * NU;
-    src = static_cast<uint32_t>(v_off_tiled(HD, false, vkey0, d)) * 4u;
+    src = I8 ? static_cast<uint32_t>(v_off_i8d(HD, vkey0, d))
+             : static_cast<uint32_t>(v_off_tiled(HD, false, vkey0, d)) * 4u;
+    scl = static_cast<uint32_t>(vkey0 * (HD / kBlock) + d / kBlock) * 4u;
+    vd = d;
     dst = static_cast<uint32_t>((kq * HD + 32 * NU * (c >> 5) + r5) * 16);
   }
   constexpr int KDST = 16 * UPR * 16, VDST = 32 * 16;
   // the loaded stage: K lanes hold unit m in r[2 m], r[2 m + 1]; V lanes key
   // e's dim in component e % 4 of r[e / 4] (NU = 1) or its two dims in half
-  // e % 2 of r[e / 2] (NU = 2).
-  float4 r[2 * NU];
-  auto load_stage = [&](int st) {
-    const size_t so = static_cast<size_t>(st) * SK * HD;
-    const auto rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>((k_stager ? kbase : vbase) + so), static_cast<short>(0), SK * HD * 4,
-        0x00020000);
+  // e % 2 of r[e / 2] (NU = 2). int8: the codes, and 8 scales in r.
+  float4 r[I8 ? 2 : 2 * NU];
+  uint32_t code[I8 ? 2 * NU : 1];
+  auto rsrc = [&](const void* at, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), static_cast<short>(0), bytes,
+                                             0x00020000);
+  };
+  auto load_codes = [&](int st) {
+    const auto rc = rsrc((k_stager ? P.k8 : P.v8) + head_el + static_cast<size_t>(st) * SK * HD, SK * HD);
     if (k_stager) {
 #pragma unroll
-      for (int i = 0; i < 2 * NU; ++i)
+      for (int m = 0; m < NU; ++m) {
+        const uint2 w = __builtin_bit_cast(
+            uint2, __builtin_amdgcn_raw_buffer_load_b64(rc, src, m * 16 * HD, 0));
+        code[2 * m] = w.x;
+        code[2 * m + 1] = w.y;
+      }
+      const auto rs = rsrc(P.ks + (static_cast<size_t>(kh) * P.ng + st) * HD, HD * 4);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        r[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, scl + 16 * i, 0, 0));
+    } else {
+#pragma unroll
+      for (int m = 0; m < NU; ++m)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          code[2 * m + i] = __builtin_amdgcn_raw_buffer_load_b32(rc, src + 16 * m + 512 * i, 0, 0);
+      constexpr int NBK = HD / kBlock;
+      const auto rs = rsrc(P.vs + (static_cast<size_t>(kh) * P.capg + st * SK) * NBK, SK * NBK * 4);
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          x[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                               rs, scl + (i + 2 * e) * NBK * 4, 0, 0));
+        r[e / 4] = make_float4(x[0], x[1], x[2], x[3]);
+      }
+    }
+  };
+  auto load_stage = [&](int st) {
+    if constexpr (I8) {
+      load_codes(st);
+      return;
+    }
+    const auto rs = rsrc((k_stager ? P.kf : P.vf) + head_el + static_cast<size_t>(st) * SK * HD, SK * HD * 4);
+    if (k_stager) {
+#pragma unroll
+      for (int i = 0; i < (I8 ? 0 : 2 * NU); ++i)
         r[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
                                               rs, src + (i & 1) * 16, (i >> 1) * 16 * HD * 4, 0));
     } else {
@@ -262,25 +329,55 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
       }
     }
   };
-  auto vdim = [&](int e, int m) -> float {
-    if constexpr (NU == 1) {
-      const float4 x = r[e / 4];
-      return e % 4 == 0 ? x.x : e % 4 == 1 ? x.y : e % 4 == 2 ? x.z : x.w;
+  auto at4 = [](const float4& x, int i) { return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w; };
+  // value e of piece m: element e of K unit m, or key e of V dim m
+  auto value = [&](int e, int m) -> float {
+    if constexpr (I8) {
+      // (code + 128) * scale - 128 * scale, rounded once: fp32(code * scale)
+      const float sc8 = at4(r[e / 4], e % 4);
+      const uint32_t w = code[2 * m + e / 4] ^ 0x80808080u;
+      return fmaf(static_cast<float>((w >> (8 * (e % 4))) & 0xFFu), sc8, -128.0f * sc8);
+    } else if (k_stager || NU == 1) {
+      return at4(r[2 * m + e / 4], e % 4);
     } else {
-      const float4 x = r[e / 2];
-      return (e & 1) == 0 ? (m == 0 ? x.x : x.y) : (m == 0 ? x.z : x.w);
+      return at4(r[e / 2], 2 * (e & 1) + m);
+    }
+  };
+  // int8: the fp32 sinks of stage st (keys < n_sink) over the lane's own
+  // stored pieces, one value at a time
+  auto put_sinks = [&](int st, int b) {
+    auto put = [&](char* at, float x) {
+      const uint32_t hi = fbits(x) & 0xFFFF0000u;
+      const float e = x - ffrom(hi);
+      const uint32_t mid = fbits(e) & 0xFFFF0000u;
+      const uint32_t part[3] = {hi, mid, fbits(e - ffrom(mid))};
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint16_t*>(at + p * PLANE) = static_cast<uint16_t>(part[p] >> 16);
+    };
+    const int t = static_cast<int>(threadIdx.x);
+#pragma unroll 1
+    for (int i = 0; i < 8 * NU; ++i) {
+      const int m = i >> 3, e = i & 7;
+      const int key = st * SK + (k_stager ? t / UPR + 16 * m : vkey0 + (e & 3) + 8 * (e >> 2));
+      if (key >= P.n_sink || key > last_key) continue;
+      const float* row = (k_stager ? P.ksink : P.vsink) + (static_cast<size_t>(kh) * P.n_sink + key) * HD;
+      put((k_stager ? kbuf(b) + m * KDST : vbuf(b) + m * VDST) + dst + 2 * e,
+          row[k_stager ? 8 * (t % UPR) + e : vd + m]);
     }
   };
   // split and store stage st into buffer b; V of keys past the workgroup's
   // last key is stored as 0 (its weight is 0, and the cache past the chunk
   // may hold anything)
   auto store_stage = [&](int st, int b) {
+    const int key0 = st * SK;
     if (k_stager) {
       char* sb = kbuf(b);
 #pragma unroll
       for (int m = 0; m < NU; ++m) {
-        const float4 lo = r[2 * m], hi = r[2 * m + 1];
-        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = value(e, m);
         uint4 part[3];
         split3(x, part);
 #pragma unroll
@@ -288,14 +385,14 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
       }
     } else {
       char* sb = vbuf(b);
-      const bool tail = st * SK + SK - 1 > last_key;  // uniform
+      const bool tail = key0 + SK - 1 > last_key;  // uniform
 #pragma unroll
       for (int m = 0; m < NU; ++m) {
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float v = vdim(e, m);
-          x[e] = !tail || st * SK + vkey0 + (e & 3) + 8 * (e >> 2) <= last_key ? v : 0.0f;
+          const float v = value(e, m);
+          x[e] = !tail || key0 + vkey0 + (e & 3) + 8 * (e >> 2) <= last_key ? v : 0.0f;
         }
         uint4 part[3];
         split3(x, part);
@@ -303,6 +400,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
         for (int p = 0; p < 3; ++p) *reinterpret_cast<uint4*>(sb + p * PLANE + m * VDST + dst) = part[p];
       }
     }
+    if (I8 && key0 < P.n_sink) put_sinks(st, b);  // uniform; rare
   };
 
   // ---- Q^T: dims 16 ks + 8 h + e of k-step ks, pre-scaled into the log2
@@ -674,10 +772,10 @@ PrefillPlan prefill_plan(const KvGeom& g, const AttnCall& c, PrefillParams* out)
   return p;
 }
 
-template <int HD>
+template <int HD, bool I8>
 hipError_t launch(const PrefillParams& p, int max_split, hipStream_t st) {
   const int items = p.n_items > 0 ? p.n_items : p.n_blocks;
-  hipLaunchKernelGGL(prefill_kernel<HD>, dim3(items * p.nkv), dim3(kPThreads), 0, st, p);
+  hipLaunchKernelGGL((prefill_kernel<HD, I8>), dim3(items * p.nkv), dim3(kPThreads), 0, st, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || max_split == 1) return e;
   constexpr int wpb = kPVec / (kMergeThreads / (HD / 4));
@@ -689,24 +787,33 @@ hipError_t launch(const PrefillParams& p, int max_split, hipStream_t st) {
 
 int prefill_split_count(const KvGeom& g, const AttnCall& c) { return prefill_plan(g, c, nullptr).max_split; }
 
-// The rows kernel streams the keys once per group of 32 vectors with little
+// The rows kernels stream the keys once per group of 32 vectors with little
 // else to pay; this kernel pays for its prologue, pipeline and merge launch
-// and then takes a quarter of the time per vector and key. Estimates in us of
-// both, from chunks of 32 to 256 rows of 8 kv heads at 0 to 8000 keys, G 1 and
-// 4 (rows | here): hd 64 G 4 64 rows at 1984 18.7 | 21.7, 100 rows 28.4 | 22.1,
-// 64 rows at 8000 45 | 39, 256 rows at 0 10.0 | 13.5, at 1984 45 | 33; hd 128
-// 64 rows at 1984 30.2 | 32.6, 100 rows 48 | 34, 128 rows at 448 25 | 23, 256
-// rows at 0 16.8 | 18.8.
+// and then takes a quarter (int8: two thirds) of the time per vector and key.
+// Estimates in us of both, from chunks of 16 to 256 rows of 8 kv heads at 0 to
+// 8000 keys, G 1, 3 and 4 (rows | here):
+//  fp32 hd 64, G 4: 64 rows at 1984 18.7 | 21.7, 100 rows 28.4 | 22.1, 64 rows
+//    at 8000 45 | 39, 256 rows at 0 10.0 | 13.5, at 1984 45 | 33;
+//  fp32 hd 128, G 4: 64 rows at 1984 30.2 | 32.6, 100 rows 48 | 34, 128 rows at
+//    448 25 | 23, 256 rows at 0 16.8 | 18.8;
+//  int8 hd 64, G 4: 100 rows at 1984 22.2 | 22.6, at 8000 56 | 46, 256 rows at
+//    448 20.9 | 19.6, at 1984 38 | 32;
+//  int8 hd 128, G 3: 100 rows at 8000 66 | 68, 256 rows at 448 30 | 26, at 1984
+//    59 | 48, at 8000 174 | 135.
 bool prefill_supported(const KvGeom& g, const AttnCall& c) {
-  if (g.int8 || g.ring || !g.tiled || c.rows < kPrefillMinRows || c.n_heads % g.nkv != 0 ||
+  if (g.ring || !g.tiled || c.rows < kPrefillMinRows || c.n_heads % g.nkv != 0 ||
       c.n_heads / g.nkv > 8)
     return false;
+  struct Cost {
+    double base, stage, split, rows, key;
+  };
+  static constexpr Cost kCost[2][2] = {{{12.0, 2.40, 0.15, 8.5, 70.5e-6}, {14.0, 4.4, 0.3, 14.0, 123e-6}},
+                                       {{10.0, 2.35, 0.15, 11.0, 52e-6}, {14.0, 4.2, 0.3, 13.0, 90e-6}}};
+  const Cost& k = kCost[g.int8][g.hd != 64];
   const int rpg = 32 / (c.n_heads / g.nkv);
-  const double groups = static_cast<double>(g.nkv) * ((c.rows + rpg - 1) / rpg);
-  const double keys = groups * (c.pos0 + c.rows / 2 + 16);
+  const double keys = static_cast<double>(g.nkv) * ((c.rows + rpg - 1) / rpg) * (c.pos0 + c.rows / 2 + 16);
   const PrefillPlan p = prefill_plan(g, c, nullptr);
-  return g.hd == 64 ? 12.0 + 2.4 * p.T + 0.15 * p.max_split < 8.5 + 70.5e-6 * keys
-                    : 14.0 + 4.4 * p.T + 0.3 * p.max_split < 14.0 + 123e-6 * keys;
+  return k.base + k.stage * p.T + k.split * p.max_split < k.rows + k.key * keys;
 }
 
 // (one region per workgroup whatever the split, so one call's workspace
@@ -722,9 +829,23 @@ hipError_t launch_prefill(const KvGeom& g, const KvStore& s, Workspace& ws, cons
   const PrefillPlan pl = prefill_plan(g, c, &p);
   if (pl.max_split > 1 && ws.part_floats < prefill_workspace_need(g, c))
     return hipErrorInvalidValue;
-  const size_t layer_el = static_cast<size_t>(c.layer) * g.nkv * head_elems(g);
-  p.kf = s.k + layer_el;
-  p.vf = s.v + layer_el;
+  const size_t layer_heads = static_cast<size_t>(c.layer) * g.nkv;
+  const size_t layer_el = layer_heads * head_elems(g);
+  if (g.int8) {
+    p.k8 = s.k8 + layer_el;
+    p.v8 = s.v8 + layer_el;
+    p.ks = s.k_scale + layer_heads * g.ngroups * g.hd;
+    p.vs = s.v_scale + layer_heads * g.capg * g.nb;
+    p.ng = g.ngroups;
+    p.n_sink = g.n_sink;
+    if (g.n_sink > 0) {
+      p.ksink = s.k_sink + layer_heads * g.n_sink * g.hd;
+      p.vsink = s.v_sink + layer_heads * g.n_sink * g.hd;
+    }
+  } else {
+    p.kf = s.k + layer_el;
+    p.vf = s.v + layer_el;
+  }
   p.q = c.q;
   p.out = c.out;
   p.part = ws.part;
@@ -737,7 +858,9 @@ hipError_t launch_prefill(const KvGeom& g, const KvStore& s, Workspace& ws, cons
   p.n_blocks = pl.n_blocks;
   p.n_items = pl.n_items;
   p.qscale = c.scale * kLog2eP;
-  return g.hd == 64 ? launch<64>(p, pl.max_split, st) : launch<128>(p, pl.max_split, st);
+  if (g.int8)
+    return g.hd == 64 ? launch<64, true>(p, pl.max_split, st) : launch<128, true>(p, pl.max_split, st);
+  return g.hd == 64 ? launch<64, false>(p, pl.max_split, st) : launch<128, false>(p, pl.max_split, st);
 }
 
 }  // namespace dbi
