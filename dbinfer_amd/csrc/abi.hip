@@ -569,27 +569,33 @@ dbi_status decode_token_impl(dbi_kv* kv, float* x, uint32_t pos) {
   return DBI_OK;
 }
 
-// decode_layer_chunk (model.cpp:933-981) from the projections: produce all n
-// rows, append them, then the causal chunk attention.
+// decode_layer_chunk (model.cpp:933-981) from the projections: one launch
+// produces and appends the n rows and ropes the queries, then the causal chunk
+// attention.
 dbi_status chunk_qkv_impl(dbi_kv* kv, uint32_t layer, uint32_t pos0, uint32_t n,
                           uint32_t n_heads, float scale, const RawQkv& r, float* out_dev) {
   if (dbi_status st = check_chunk(kv, pos0, n)) return st;
   if (n == 0) return DBI_OK;
   if (dbi_status st = ensure_rope_table(kv)) return st;
-  const size_t qn = size_t(n) * n_heads * kv->geom.hd;
-  const size_t kn = size_t(n) * kv->geom.nkv * kv->geom.hd;
-  if (dbi_status st = ensure_prod(kv, qn + 2 * kn)) return st;
+  if (dbi_status st = ensure_prod(kv, size_t(n) * n_heads * kv->geom.hd)) return st;
   float* qo = kv->ws.prod;
-  float* ko = qo + qn;
-  float* vo = ko + kn;
   const dbi::AttnCall c = chunk_call(layer, pos0, n, n_heads, scale, qo, out_dev);
   bool prefill = false;
   if (dbi_status st = chunk_prepare(kv, c, &prefill)) return st;
-  const dbi::ProduceCall pc{static_cast<int>(n), static_cast<int>(pos0),
-                            static_cast<int>(n_heads), r.q, r.k, r.v, r.qb, r.kb, r.vb,
-                            qo, ko, vo};
-  HIP_TRY(dbi::launch_produce(kv->geom, kv->store.rope_dd, pc, kv->stream), "producer launch");
-  if (dbi_status st = append_impl(kv, layer, pos0, n, ko, vo)) return st;
+  dbi::AppendRows a{};
+  a.k = r.k;
+  a.v = r.v;
+  a.kb = r.kb;
+  a.vb = r.vb;
+  a.cs = kv->store.rope_dd;
+  a.q = r.q;
+  a.qb = r.qb;
+  a.q_out = qo;
+  a.n_heads = static_cast<int>(n_heads);
+  HIP_TRY(dbi::launch_append_rows(kv->geom, kv->store, static_cast<int>(layer),
+                                  static_cast<int>(pos0), static_cast<int>(n), a, kv->stream),
+          "append launch");
+  kv->n_seen = pos0 + n;
   return chunk_launch(kv, c, prefill);
 }
 

@@ -190,6 +190,32 @@ struct AttnCall {
 // Launchers (return a hipError_t of the launch).
 hipError_t launch_append(const KvGeom& g, const KvStore& s, int layer, int pos0, int n,
                          const float* k, const float* v, hipStream_t st);
+// The same for a dense cache of head dim 64 or 128, from raw projections: k, v
+// [n][nkv*hd] plus the biases (or null), K roped with the (cos, sin) table cs
+// [cap][hd/2] (null: as it is); with q [n][n_heads*hd] the biased, roped
+// queries go to q_out. One launch.
+struct AppendRows {
+  const float* k;
+  const float* v;
+  const float* kb;
+  const float* vb;
+  const double2* cs;
+  const float* q;
+  const float* qb;
+  float* q_out;  // 16-byte aligned
+  int n_heads;
+};
+hipError_t launch_append_rows(const KvGeom& g, const KvStore& s, int layer, int pos0, int n,
+                              const AppendRows& r, hipStream_t st);
+
+// fp64 rotation of one NeoX pair (tensor::rope, ops.cpp:19-38), each product
+// and sum rounded on its own
+__device__ __forceinline__ float2 rope_rotate(float a, float b, double c, double s) {
+#pragma clang fp contract(off)
+  const double x = static_cast<double>(a) * c - static_cast<double>(b) * s;
+  const double y = static_cast<double>(b) * c + static_cast<double>(a) * s;
+  return make_float2(static_cast<float>(x), static_cast<float>(y));
+}
 // Returns hipErrorNotSupported for shapes without a kernel instance.
 hipError_t launch_attention(const KvGeom& g, const KvStore& s, Workspace& ws,
                             const AttnCall& c, hipStream_t st);

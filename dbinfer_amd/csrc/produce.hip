@@ -39,14 +39,6 @@ struct ProduceArgs {
   int rows, nh, nkv, hd, pos0;
 };
 
-// fp64 rotation of one NeoX pair, each product and sum rounded on its own
-__device__ __forceinline__ float2 rotate(float a, float b, double c, double s) {
-#pragma clang fp contract(off)
-  const double x = static_cast<double>(a) * c - static_cast<double>(b) * s;
-  const double y = static_cast<double>(b) * c + static_cast<double>(a) * s;
-  return make_float2(static_cast<float>(x), static_cast<float>(y));
-}
-
 // One thread per pair (j, j + hd/2) of one head of one row: the nh query
 // heads, then the nkv key heads, then the nkv value heads (bias only).
 // Consecutive threads take consecutive j, so each half-row is one coalesced
@@ -92,7 +84,7 @@ __global__ __launch_bounds__(kThreads) void produce_kernel(ProduceArgs a) {
   }
   if (a.cs != nullptr && h < a.nh + a.nkv) {
     const double2 t = a.cs[static_cast<size_t>(a.pos0 + r) * half + j];
-    const float2 y = rotate(x0, x1, t.x, t.y);
+    const float2 y = rope_rotate(x0, x1, t.x, t.y);
     x0 = y.x;
     x1 = y.y;
   }
