@@ -78,6 +78,7 @@ void free_store(dbi::KvStore& s) {
 void free_ws(dbi::Workspace& w) {
   if (w.part) (void)hipFree(w.part);
   if (w.pinned) (void)hipHostFree(w.pinned);
+  if (w.box) (void)hipHostFree(w.box);
   if (w.counters) (void)hipFree(w.counters);
   if (w.staging) (void)hipFree(w.staging);
   if (w.prod) (void)hipFree(w.prod);
@@ -96,6 +97,65 @@ dbi_status need_staging(dbi_kv* kv, size_t floats) {
   kv->ws.staging_floats = floats;
   return DBI_OK;
 }
+
+// The rows of one single-row host call on their way to the device and back:
+// the inputs are gathered in a pinned box of the handle, one small kernel
+// fetches them, and the attention kernel stores its output into the box. (A
+// copy call per row of pageable memory, each staged by the runtime, and one
+// back took 40 us of such a call's time against 8 of the attention kernel.)
+class HostRows {
+ public:
+  HostRows(dbi_kv* kv, size_t in_floats, size_t out_floats)
+      : kv_(kv), in_(round4(in_floats)), out_(round4(out_floats)) {}
+  static size_t round4(size_t n) { return (n + 3) & ~size_t(3); }
+  // room for both; every row starts 16-byte aligned (sizes rounded up)
+  dbi_status open() {
+    dbi::Workspace& w = kv_->ws;
+    if (w.box_floats < in_ + out_) {
+      if (w.box) (void)hipHostFree(w.box);
+      w.box = w.box_dev = nullptr;
+      w.box_floats = 0;
+      void* p = nullptr;
+      void* d = nullptr;
+      if (hipHostMalloc(&p, (in_ + out_) * sizeof(float), hipHostMallocMapped) != hipSuccess)
+        return fail(DBI_ERR_NOMEM, "out of pinned host memory for a host call's rows");
+      if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
+        (void)hipHostFree(p);
+        return fail(DBI_ERR_DEVICE, "pinned host memory is not mapped");
+      }
+      w.box = static_cast<float*>(p);
+      w.box_dev = static_cast<float*>(d);
+      w.box_floats = in_ + out_;
+    }
+    return need_staging(kv_, in_);
+  }
+  // the row's device address after fetch(); null stays null
+  const float* add(const float* src, size_t n) {
+    if (src == nullptr) return nullptr;
+    std::memcpy(kv_->ws.box + at_, src, n * sizeof(float));
+    const float* dev = kv_->ws.staging + at_;
+    at_ += round4(n);
+    return dev;
+  }
+  float* out_dev() const { return kv_->ws.box_dev + in_; }
+  dbi_status fetch() {
+    HIP_TRY(dbi::launch_fetch(kv_->ws.box_dev, kv_->ws.staging, at_, kv_->stream), "row fetch");
+    return DBI_OK;
+  }
+  // after the step: its output into the caller's row, or after a failed one
+  // only the wait (the box is free again)
+  dbi_status close(dbi_status st, float* out, size_t n) {
+    const hipError_t e = hipStreamSynchronize(kv_->stream);
+    if (st != DBI_OK) return st;
+    if (e != hipSuccess) return hip_fail(e, "stream sync");
+    std::memcpy(out, kv_->ws.box + in_, n * sizeof(float));
+    return DBI_OK;
+  }
+
+ private:
+  dbi_kv* kv_;
+  size_t in_, out_, at_ = 0;
+};
 
 dbi_status check_layer(const dbi_kv* kv, uint32_t layer) {
   if (layer >= kv->cfg.n_layers)
@@ -607,6 +667,15 @@ dbi_status qkv_host(dbi_kv* kv, uint32_t layer, uint32_t pos0, uint32_t n, uint3
   if (n == 0) return chunk ? check_chunk(kv, pos0, n) : DBI_OK;
   const size_t hq = size_t(n_heads) * kv->geom.hd, hk = size_t(kv->geom.nkv) * kv->geom.hd;
   const size_t qn = n * hq, kn = n * hk;
+  if (!chunk) {
+    HostRows rows(kv, 2 * HostRows::round4(hq) + 4 * HostRows::round4(hk), hq);
+    if (dbi_status st = rows.open()) return st;
+    const RawQkv d{rows.add(h.q, hq), rows.add(h.k, hk), rows.add(h.v, hk),
+                   rows.add(h.qb, hq), rows.add(h.kb, hk), rows.add(h.vb, hk)};
+    dbi_status st = rows.fetch();
+    if (st == DBI_OK) st = decode_qkv_impl(kv, layer, pos0, n_heads, scale, d, rows.out_dev());
+    return rows.close(st, out, hq);
+  }
   const size_t need = 2 * qn + 2 * kn + (h.qb ? hq : 0) + (h.kb ? hk : 0) + (h.vb ? hk : 0);
   if (dbi_status st = need_staging(kv, need)) return st;
   float* at = kv->ws.staging;
@@ -626,8 +695,7 @@ dbi_status qkv_host(dbi_kv* kv, uint32_t layer, uint32_t pos0, uint32_t n, uint3
   HIP_TRY(up(h.kb, hk, &d.kb), "k bias upload");
   HIP_TRY(up(h.vb, hk, &d.vb), "v bias upload");
   float* od = at;
-  const dbi_status st = chunk ? chunk_qkv_impl(kv, layer, pos0, n, n_heads, scale, d, od)
-                              : decode_qkv_impl(kv, layer, pos0, n_heads, scale, d, od);
+  const dbi_status st = chunk_qkv_impl(kv, layer, pos0, n, n_heads, scale, d, od);
   if (st != DBI_OK) {
     (void)hipStreamSynchronize(kv->stream);  // the uploads read the caller's buffers
     return st;
@@ -902,16 +970,12 @@ dbi_status dbi_attn_decode(dbi_kv* kv, uint32_t layer, uint32_t pos, uint32_t n_
   if (kv == nullptr) return fail(DBI_ERR_INVALID, "null handle");
   if (dbi_status st = check_attend(kv, layer, n_heads, q, out)) return st;
   const size_t elems = size_t(n_heads) * kv->cfg.head_dim;
-  if (dbi_status st = need_staging(kv, 2 * elems)) return st;
-  float* qd = kv->ws.staging;
-  float* od = kv->ws.staging + elems;
-  HIP_TRY(hipMemcpyAsync(qd, q, elems * sizeof(float), hipMemcpyHostToDevice, kv->stream),
-          "copy q");
-  if (dbi_status st = decode_impl(kv, layer, pos, n_heads, scale, qd, od)) return st;
-  HIP_TRY(hipMemcpyAsync(out, od, elems * sizeof(float), hipMemcpyDeviceToHost, kv->stream),
-          "copy out");
-  HIP_TRY(hipStreamSynchronize(kv->stream), "attention sync");
-  return DBI_OK;
+  HostRows rows(kv, elems, elems);
+  if (dbi_status st = rows.open()) return st;
+  const float* qd = rows.add(q, elems);
+  dbi_status st = rows.fetch();
+  if (st == DBI_OK) st = decode_impl(kv, layer, pos, n_heads, scale, qd, rows.out_dev());
+  return rows.close(st, out, elems);
 }
 
 dbi_status dbi_attn_decode_async(dbi_kv* kv, uint32_t layer, uint32_t pos, uint32_t n_heads,
@@ -946,18 +1010,14 @@ dbi_status dbi_kv_decode(dbi_kv* kv, uint32_t layer, uint32_t pos, const float* 
   if (dbi_status st = check_attend(kv, layer, n_heads, q, out)) return st;
   const size_t P = size_t(kv->cfg.n_kv_heads) * kv->cfg.head_dim;
   const size_t qn = size_t(n_heads) * kv->cfg.head_dim;
-  if (dbi_status st = need_staging(kv, 2 * P + 2 * qn)) return st;
-  float* kd = kv->ws.staging;
-  float* vd = kd + P;
-  float* qd = vd + P;
-  float* od = qd + qn;
-  HIP_TRY(hipMemcpyAsync(kd, k, P * 4, hipMemcpyHostToDevice, kv->stream), "k upload");
-  HIP_TRY(hipMemcpyAsync(vd, v, P * 4, hipMemcpyHostToDevice, kv->stream), "v upload");
-  HIP_TRY(hipMemcpyAsync(qd, q, qn * 4, hipMemcpyHostToDevice, kv->stream), "q upload");
-  if (dbi_status st = decode_impl(kv, layer, pos, n_heads, scale, qd, od, kd, vd)) return st;
-  HIP_TRY(hipMemcpyAsync(out, od, qn * 4, hipMemcpyDeviceToHost, kv->stream), "out readback");
-  HIP_TRY(hipStreamSynchronize(kv->stream), "stream sync");
-  return DBI_OK;
+  HostRows rows(kv, 2 * HostRows::round4(P) + qn, qn);
+  if (dbi_status st = rows.open()) return st;
+  const float* kd = rows.add(k, P);
+  const float* vd = rows.add(v, P);
+  const float* qd = rows.add(q, qn);
+  dbi_status st = rows.fetch();
+  if (st == DBI_OK) st = decode_impl(kv, layer, pos, n_heads, scale, qd, rows.out_dev(), kd, vd);
+  return rows.close(st, out, qn);
 }
 
 dbi_status dbi_kv_decode_async(dbi_kv* kv, uint32_t layer, uint32_t pos, const float* k_dev,

@@ -147,6 +147,9 @@ struct Workspace {
   float* staging = nullptr;  // device staging for host-pointer calls
   unsigned char* pinned = nullptr;  // pinned host chunk for prefix-file transfers
   size_t staging_floats = 0;
+  float* box = nullptr;      // pinned host rows of single-row host calls, as the host sees them
+  float* box_dev = nullptr;  // and as kernels do
+  size_t box_floats = 0;
   float* prod = nullptr;  // producer output: roped q, roped k, biased v rows
   size_t prod_floats = 0;
   // verify round: slice keys, arrival counter and the host variant's token
@@ -260,6 +263,8 @@ struct ProduceCall {
   float* k_out;
   float* v_out;
 };
+// n floats (a multiple of 4, 16-byte aligned) from mapped host memory
+hipError_t launch_fetch(const float* src, float* dst, size_t n, hipStream_t st);
 hipError_t launch_produce(const KvGeom& g, const double2* rope_dd, const ProduceCall& c,
                           hipStream_t st);
 // Host table of (cos, sin) for every position < cap and pair of the head

@@ -92,7 +92,25 @@ __global__ __launch_bounds__(kThreads) void produce_kernel(ProduceArgs a) {
   dst[at + half] = x1;
 }
 
+// One 16-byte piece a thread, every load of the rows in flight at once: a
+// decode step's ~10 KB take one PCIe round trip.
+__global__ __launch_bounds__(kThreads) void fetch_kernel(const float4* __restrict__ src,
+                                                         float4* __restrict__ dst, unsigned n4) {
+  const unsigned i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n4) dst[i] = src[i];
+}
+
 }  // namespace
+
+hipError_t launch_fetch(const float* src, float* dst, size_t n, hipStream_t st) {
+  const size_t n4 = n / 4;
+  if (n4 == 0) return hipSuccess;
+  if (n % 4 != 0 || n4 > (size_t(1) << 30)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(fetch_kernel, dim3(static_cast<unsigned>((n4 + kThreads - 1) / kThreads)),
+                     dim3(kThreads), 0, st, reinterpret_cast<const float4*>(src),
+                     reinterpret_cast<float4*>(dst), static_cast<unsigned>(n4));
+  return hipGetLastError();
+}
 
 bool rope_table_host(const KvGeom& g, float theta, double2* tab) {
   if (g.hd < 2 || g.hd % 2 != 0) return false;
