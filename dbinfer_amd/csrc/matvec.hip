@@ -59,6 +59,8 @@ struct MvArgs {
   int seg_end[3];       // plain: cumulative row ends of the segments
   int rows;             // plain: total rows; pair: rows of each matrix
   int tasks, chunks;    // tasks of kNR row dots; units per task
+  int per, extra;       // tasks per workgroup, one more for the first `extra`
+  int batch;            // tasks per batch
   int pair, acc;
 };
 
@@ -76,12 +78,6 @@ typedef __attribute__((address_space(1))) const float gf32;
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const f4v gf4;
 typedef __attribute__((address_space(1))) float gf32w;
-
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
 
 __device__ inline uint32_t pack4(int8_t a, int8_t b, int8_t c, int8_t d) {
   return static_cast<uint32_t>(static_cast<uint8_t>(a)) |
@@ -106,6 +102,27 @@ __device__ __forceinline__ float dpp_add(float v, int ctrl) {
     default:
       return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
   }
+}
+
+// Sum over the wave, in every lane: DPP inside a row of 16, then the four rows'
+// sums by lane reads (six ds_bpermute steps took ~0.3 us of a launch).
+__device__ __forceinline__ float wave_sum(float v) {
+  v = dpp_add(v, 0xB1);
+  v = dpp_add(v, 0x4E);
+  v = dpp_add(v, 0x141);
+  v = dpp_add(v, 0x140);
+  auto row = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+  return (row(0) + row(16)) + (row(32) + row(48));
+}
+
+// Lane halves exchanged: a keeps its lower half and takes b's lower half as its
+// upper one, b the upper halves (the rows of 16: odd rows of a, even of b).
+// Through asm: the builtins fold the two results into one when both are used.
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
 
 // The row pointers of task t's row dots.
@@ -213,11 +230,13 @@ __device__ __forceinline__ void sum_row(const uint32_t w[Pair<Q4>::kDw], const A
 // A unit's kNR lane sums, reduced together: two halving steps leave lane l
 // with a partial of row l >> 4, four in-row DPP steps finish it; lane 16r
 // returns row r's sum.
-__device__ inline float reduce_unit(const float acc[kNR], int lane) {
-  const bool h5 = lane >= 32, h4 = (lane & 16) != 0;
-  const float b0 = (h5 ? acc[2] : acc[0]) + __shfl_xor(h5 ? acc[0] : acc[2], 32);
-  const float b1 = (h5 ? acc[3] : acc[1]) + __shfl_xor(h5 ? acc[1] : acc[3], 32);
-  float v = (h4 ? b1 : b0) + __shfl_xor(h4 ? b0 : b1, 16);
+__device__ inline float reduce_unit(const float acc[kNR]) {
+  float a0 = acc[0], a1 = acc[1], a2 = acc[2], a3 = acc[3];
+  swap32(a0, a2);
+  swap32(a1, a3);
+  float b0 = a0 + a2, b1 = a1 + a3;
+  swap16(b0, b1);
+  float v = b0 + b1;
   v = dpp_add(v, 0xB1);   // quad_perm [1,0,3,2]
   v = dpp_add(v, 0x4E);   // quad_perm [2,3,0,1]
   v = dpp_add(v, 0x141);  // row_half_mirror
@@ -412,9 +431,12 @@ __global__ __launch_bounds__(kMvThreads) void matvec_q_kernel(const MvArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int C = a.chunks;
-  const int t0 = static_cast<int>(static_cast<long long>(a.tasks) * blockIdx.x / gridDim.x);
-  const int t1 = static_cast<int>(static_cast<long long>(a.tasks) * (blockIdx.x + 1) / gridDim.x);
-  const int bt = max(1, kBatchUnits / C);  // tasks per batch
+  // (the shares are divided on the host: here, in 64 bits, that alone took
+  // 1 us of every launch before its first load)
+  const int wg = static_cast<int>(blockIdx.x);
+  const int t0 = wg * a.per + min(wg, a.extra);
+  const int t1 = t0 + a.per + (wg < a.extra ? 1 : 0);
+  const int bt = a.batch;
   RowHold h;
   hold_row(a, h);
   uint32_t wd[kNR][Pair<Q4>::kDw];
@@ -426,6 +448,7 @@ __global__ __launch_bounds__(kMvThreads) void matvec_q_kernel(const MvArgs a) {
   // registers, so every wave keeps about kNR rows in flight without a second
   // register set. The first unit is requested before the activation
   // prologue.
+  auto unit_task = [&](int u) { return C == 1 ? u : u / C; };
   auto batch_units = [&](int tb) { return min(bt, t1 - tb) * C; };
   int ltb = t0, lu = wave;  // the unit in flight
   auto next = [&]() {  // false: the wave has no further unit
@@ -442,7 +465,7 @@ __global__ __launch_bounds__(kMvThreads) void matvec_q_kernel(const MvArgs a) {
   };
   auto first_load = [&]() {
     if (wave < batch_units(t0)) {
-      const int k = lu / C;
+      const int k = unit_task(lu);
       task_rows<Q4>(a, ltb + k, wr);
 #pragma unroll
       for (int r = 0; r < kNR; ++r) load_row<Q4>(wd[r], wr[r], lu - k * C, a.npair, lane);
@@ -464,9 +487,9 @@ __global__ __launch_bounds__(kMvThreads) void matvec_q_kernel(const MvArgs a) {
 #pragma unroll 1
     for (int u = wave; u < nu; u += kMvWaves) {
       ActPair x;
-      load_act<Q4>(x, u % C, a.npair, lane, s_code, s_dx, s_sum);
+      load_act<Q4>(x, u - unit_task(u) * C, a.npair, lane, s_code, s_dx, s_sum);
       const bool more = next();  // wave-uniform
-      const int nk = lu / C, nc = lu - nk * C;
+      const int nk = unit_task(lu), nc = lu - nk * C;
       task_rows<Q4>(a, ltb + nk, wr);
       float acc[kNR];
 #pragma unroll
@@ -475,7 +498,7 @@ __global__ __launch_bounds__(kMvThreads) void matvec_q_kernel(const MvArgs a) {
         sum_row<Q4>(wd[r], x, acc[r]);
         if (more) load_row<Q4>(wd[r], wr[r], nc, a.npair, lane);
       }
-      const float v = reduce_unit(acc, lane);
+      const float v = reduce_unit(acc);
       if (C == 1) {
         // a unit is a whole task: lane 16r holds row r (for pairs, up row r
         // sits in lane 16r + 32)
@@ -550,6 +573,9 @@ hipError_t launch_matvec_q(const MatvecCall& c, hipStream_t st) {
   const int grid = static_cast<int>(
       min(static_cast<long long>((a.chunks > 1 ? 1 : kWgPerCu) * ncu),
           max(static_cast<long long>(min(ncu, a.tasks)), (units + kMvWaves - 1) / kMvWaves)));
+  a.per = a.tasks / grid;
+  a.extra = a.tasks % grid;
+  a.batch = kBatchUnits / a.chunks > 1 ? kBatchUnits / a.chunks : 1;
   const size_t lds = static_cast<size_t>(a.nbk) * (c.q4 ? 10 : 9) * sizeof(uint32_t);
   if (c.q4)
     hipLaunchKernelGGL(matvec_q_kernel<true>, dim3(grid), dim3(kMvThreads), lds, st, a);
