@@ -492,9 +492,19 @@ __global__ __launch_bounds__(kRowThreads) void rows_i8_kernel(KvGeom g, KvStore 
     for (int i = tid; i < CH / 16; i += kRowThreads)
       reinterpret_cast<f4a*>(v8)[i] = reinterpret_cast<const f4a*>(s_v)[i];
   } else {
-    for (int i = tid; i < CH; i += kRowThreads) {
-      const int w = 16 * ((i >> 2) & 1) + 4 * ((i >> 8) & 3) + (i & 3);
-      if (w >= vlo && w <= within) v8[i] = s_v[i];
+    // 4 bytes: a channel of positions w .. w + 3
+#pragma unroll
+    for (int i = tid; i < CH / 4; i += kRowThreads) {
+      const int w = 16 * (i & 1) + 4 * ((i >> 6) & 3);
+      if (w + 3 < vlo || w > within) continue;
+      const uint32_t x = reinterpret_cast<const uint32_t*>(s_v)[i];
+      if (w >= vlo && w + 3 <= within) {
+        reinterpret_cast<uint32_t*>(v8)[i] = x;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (w + j >= vlo && w + j <= within) v8[4 * i + j] = static_cast<int8_t>(x >> (8 * j));
+      }
     }
   }
   // ---- the staging rows after the batch
