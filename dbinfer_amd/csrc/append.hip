@@ -234,7 +234,8 @@ __global__ __launch_bounds__(kThreads) void rows_pack_kernel(const float* store,
 // are each other's rope partners (dims 4 c.. and hd/2 + 4 c..: a granule's
 // layout), a V piece dims 8 c.. .
 // Measured, a layer's whole chunk step: 5 rows at 16 k (32/8 heads, hd 128)
-// int8 37.8 -> 27.6 us, fp32 35.5 -> 33.2; 256 int8 rows at 3840 99.7 -> 88.0;
+// int8 37.8 -> 27.1 us (0.4 of it V codes in 4-byte stores; twice the threads
+// at hd 128 measured no faster), fp32 35.5 -> 33.2; 256 int8 rows at 3840 99.7 -> 88.0;
 // 1000 fp32 rows of 28/4 heads 75.5 -> 70.7.
 constexpr int kRowThreads = 256;
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // rows of any alignment
